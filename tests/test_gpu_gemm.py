@@ -112,3 +112,44 @@ def test_gemm(hip, oc, fmt, M, N, K):
     err = rel_l2(got - y0, ref - y0)
     print(f"fmt {fmt} M {M} N {N} K {K}: rel_l2 {err:.2e}")
     assert err < 1e-5
+
+
+# Edges of the 16-, 32- and 64-wide tiles, one chunk to a few per wave (Q4_K: empty K quarters at K = 256), and
+# M x N on both sides of where the tile changes: Q8_0 at 512 tiles of 16 x 32, 1216 and 8192 of 32 x 32; Q4_K at 768
+# tiles of 32 x 64 and 1280 of 64 x 64 whose tokens fill them.
+EDGES = [(m, n, k) for m, n in ((1, 7), (16, 33), (17, 16), (31, 65), (33, 31), (64, 64), (65, 17))
+         for k in (256, 512, 1280)]
+EDGES += [(m, n, 256) for m, n in ((16, 16384 - 33), (16, 16384 - 31), (33, 608 * 32 - 33), (33, 608 * 32 - 31),
+                                   (100, 65536 - 33), (100, 65536 - 31), (32, 49152 - 65), (32, 49152 - 63),
+                                   (64, 81920 - 65), (64, 81920 - 63), (80, 41000), (352, 12352))]
+
+
+@pytest.mark.parametrize("fmt", (Q8_0, Q4_K))
+@pytest.mark.parametrize("M,N,K", EDGES)
+def test_gemm_edges(hip, oc, fmt, M, N, K):
+    """Against exact products of the quantized operands: K/32 fp32 roundings of block products and as many of the
+    running sum, each within 2^-24 of a sum that is at most a few times the result, so under 1e-6 relative L2 for
+    K <= 1280 (a lost block or scale is 1e-1).  The rest of y's row (ldy > N) is not touched, and a token's row is
+    the same bits alone as among M tokens, whatever tile each takes."""
+    import torch
+    gguf = synth.q8_0_blocks(41, min(N, 512), K) if fmt == Q8_0 else synth.q4_K_blocks(42, min(N, 512), K)
+    W = np.tile(gguf, (-(-N // len(gguf)), 1))[:N]
+    X = (synth.activations(43, M * K) * 2.0).astype(np.float32).reshape(M, K)
+    tiled = empty(hip.tiled_bytes(fmt, N, K), torch.uint8)
+    hip.repack(fmt, dev(W), tiled, N, K)
+
+    def product(x):
+        act = empty(hip.gemm_act_bytes(fmt, len(x), K), torch.uint8)
+        hip.gemm_quantize_act(fmt, dev(x), act, len(x), K)
+        y = dev(np.full((len(x), N + 3), 9.0, np.float32))
+        hip.gemm(fmt, tiled, act, y, len(x), N, K, ldy=N + 3)
+        return host(y)
+    got = product(X)
+    assert (got[:, N:] == 9.0).all()
+    Wd = q8_dequant(gguf, K) if fmt == Q8_0 else q4k_dequant(gguf, K)
+    ref = np.tile(x_dequant(oc, fmt, X) @ Wd.T, (1, -(-N // len(gguf))))[:, :N]
+    err = rel_l2(got[:, :N], ref)
+    print(f"fmt {fmt} M {M} N {N} K {K}: rel_l2 {err:.2e}")
+    assert err < 1e-6
+    for m in {0, M - 1}:
+        assert np.array_equal(product(X[m:m + 1])[0], got[m])
