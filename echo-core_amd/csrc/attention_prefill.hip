@@ -10,7 +10,7 @@
 // head (32 query rows) and walks the key blocks of 64 positions up to its last
 // token once: each block's K and V bytes are staged in LDS a single time for
 // all 32 rows (V transposed to [dim][position]).  Scores and softmax . V run
-// on v_mfma_i32_16x16x32_i8 as in the decode kernel: q and (probability x V
+// on v_mfma_i32_16x16x64_i8 as in the decode kernel: q and (probability x V
 // row scale) are each split into three int8 pieces (layout.hpp split_pieces),
 // so every product is an exact int32 and the pieces recombine in fp32.  The
 // A rows of a 16-row MFMA tile are 4 query rows x 4 piece slots (the fourth
@@ -59,16 +59,15 @@ __host__ __device__ inline uint32_t prefill_segments(uint32_t positions) {
 }
 
 struct PrefillLds {
-    uint8_t K[kKb][kKs];
-    uint32_t vT[kHd * kVs + 2 * (kHd / 16)];  // [dim][position quad], rows skewed (vt_at)
+    uint8_t K[2][kKb][kKs];                      // by block parity
+    uint32_t vT[2][kHd * kVs + 2 * (kHd / 16)];  // [dim][position quad], rows skewed (vt_at)
     uint8_t P[kRows / 4][16][kPs];    // per row tile: [4 query rows x 4 piece slots][position]
     uint8_t q[kRows][kQPieces][kHd];  // q pieces of the workgroup's query rows
     float qs[kRows][4];               // piece steps (slot 3 unused)
-    float ks[kKb], vs[kKb];
-    float vsw[4];  // per-wave maxima of the V row scales
+    float ks[2][kKb], vs[2][kKb];
+    float vsw[8];         // per-wave maxima of the V row scales
+    uint32_t rise[2][8];  // per block parity and wave: a row maximum rises in this block
 };
-
-__device__ __forceinline__ long pack2(uint32_t lo, uint32_t hi) { return (long)(((uint64_t)hi << 32) | (uint64_t)lo); }
 
 __device__ __forceinline__ float row16_max(float v) {
     v = fmaxf(v, lane_xor<1>(v));
@@ -81,15 +80,27 @@ __device__ __forceinline__ float row16_max(float v) {
 }  // namespace
 
 // grid 8 * ceil(nqb * n_kv / 8) (nqb = ceil(T / (32/G)) query blocks), block
-// 256.  Workgroups are dispatched to the 8 XCDs round-robin (blockIdx % 8);
+// 512.  Workgroups are dispatched to the 8 XCDs round-robin (blockIdx % 8);
 // XCD x takes the contiguous (kv head, query block) range [x*per, (x+1)*per)
 // in kv-head-major order, so each XCD's L2 holds the K/V rows of one or two
 // kv heads instead of all of them (every query block re-reads its kv head's
 // cache).  Query row r (0 .. 31) is token r/G of the workgroup's QB tokens
-// and head kvh + n_kv*(r%G); row tile i (8 of them) holds query rows
-// 4i .. 4i+3, wave w owns tiles 2w and 2w+1.
+// and head kvh + n_kv*(r%G); wave w owns row tile w, query rows 4w .. 4w+3.
+//
+// What bounds it: instruction issue.  A block is about 400 VALU operations, 32
+// MFMAs and 36 LDS operations per wave in one dependent chain, and a wave alone
+// issues a VALU operation every 5 clocks, two waves one every 2.5: so eight
+// waves of one row tile each, two per SIMD, rather than four of two.  A pair of
+// waves (rows 8i .. 8i+7) flushes together, when a maximum of either rises: the
+// sums are then the same bits as with one wave for both tiles.  K and V are
+// double-buffered, and a block's scores are formed while the block before goes
+// through softmax . V: one barrier per block, which also carries the rises.
+// 512 tokens at 3584, 16 / 4 heads: 227 us with four waves of two tiles and
+// 16x16x32 products, 161 with eight waves, 16x16x64 products and single
+// buffers (two barriers a block), 150 as it is; the floor of its int8 products
+// and bytes is about 28.
 template <int G>
-__global__ __launch_bounds__(256) void k_attn_prefill(const float* __restrict__ q, const int8_t* __restrict__ keys,
+__global__ __launch_bounds__(512, 2) void k_attn_prefill(const float* __restrict__ q, const int8_t* __restrict__ keys,
                                                       const int8_t* __restrict__ vals,
                                                       const float* __restrict__ kscales,
                                                       const float* __restrict__ vscales, float* __restrict__ out,
@@ -101,7 +112,8 @@ __global__ __launch_bounds__(256) void k_attn_prefill(const float* __restrict__ 
     const uint32_t wg = (blockIdx.x % 8) * per + blockIdx.x / 8;
     if (wg >= total) return;  // grid padding (whole workgroup, before any barrier)
     const uint32_t kvh = wg / (nqb * S), qb = (wg / S) % nqb, seg = wg % S;
-    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6, r16 = lane & 15, g4 = lane >> 4;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, r16 = lane & 15, g4 = lane >> 4;
+    const uint32_t w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t n_heads = n_kv * G;
     const uint32_t t_first = qb * QB, n_tok = min(QB, T - t_first);
     const uint32_t last_pos = pos0 + t_first + n_tok - 1;
@@ -112,8 +124,8 @@ __global__ __launch_bounds__(256) void k_attn_prefill(const float* __restrict__ 
     const int8_t* kb = keys + (size_t)kvh * kHd;
     const int8_t* vb = vals + (size_t)kvh * kHd;
 
-    // ---- q pieces of the 32 rows: wave w packs rows 8w .. 8w+7, lane = 4 dims
-    for (uint32_t r = 8 * w; r < 8 * w + 8; ++r) {
+    // ---- q pieces of the 32 rows: wave w packs rows 4w .. 4w+3, lane = 4 dims
+    for (uint32_t r = 4 * w; r < 4 * w + 4; ++r) {
         const uint32_t tq = r / G, head = kvh + n_kv * (r % G);
         float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
         if (tq < n_tok) v4 = *(const float4*)(q + ((size_t)(t_first + tq) * n_heads + head) * kHd + 4 * lane);
@@ -134,182 +146,179 @@ __global__ __launch_bounds__(256) void k_attn_prefill(const float* __restrict__ 
         if (lane == 0) *(float4*)&L.qs[r][0] = make_float4(steps[0], steps[1], steps[2], 0.f);
     }
 
-    // ---- staging of key block b: K rows (thread = 16 bytes of one row) and V
-    // transposed (thread = 16 dims x positions kq, kq+16, kq+32, kq+48 of the
+    // ---- staging of key block b: K rows (thread = 16 bytes of two rows) and V
+    // transposed (thread = 8 dims x positions kq, kq+16, kq+32, kq+48 of the
     // block, 4x4 byte transposes): softmax . V contracts over the index
     // 4*(position % 16) + position / 16, so that a lane's four probabilities
     // (its position in each 16-position key tile) form one LDS dword.
     // Positions past last_pos repeat last_pos (masked in the scores).
-    u32x4 kr[4], vr[4];
+    u32x4 kr[2];
+    uint2 vr[4];
     float ksr = 0.f, vsr = 0.f;
-    auto load = [&](uint32_t b) {
-        const uint32_t p0 = b * kKb;
+    const uint32_t kc = tid % 16, kk = tid / 16, dg = tid % 32, kq = tid / 32;
+    auto load_k = [&](uint32_t b) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t i = tid + 256 * j, key = i / 16, c = i % 16;
-            const uint32_t p = min(p0 + key, last_pos);
-            kr[j] = *(const u32x4*)(kb + (size_t)p * row + 16 * c);
-        }
-        const uint32_t dg = tid % 16, kq = tid / 16;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t p = min(p0 + kq + 16 * j, last_pos);
-            vr[j] = *(const u32x4*)(vb + (size_t)p * row + 16 * dg);
-        }
-        if (tid < kKb) {
-            const uint32_t p = min(p0 + tid, last_pos);
-            ksr = kscales[(size_t)p * n_kv + kvh];
-            vsr = vscales[(size_t)p * n_kv + kvh];
-        }
+        for (int j = 0; j < 2; ++j)
+            kr[j] = *(const u32x4*)(kb + (size_t)min(b * kKb + kk + 32 * j, last_pos) * row + 16 * kc);
+        if (tid < kKb) ksr = kscales[(size_t)min(b * kKb + tid, last_pos) * n_kv + kvh];
     };
-    auto store = [&]() {
+    auto load_v = [&](uint32_t b) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const uint32_t i = tid + 256 * j, key = i / 16, c = i % 16;
-            *(u32x4*)&L.K[key][16 * c] = kr[j];
-        }
-        const uint32_t dg = tid % 16, kq = tid / 16;
+        for (int j = 0; j < 4; ++j)
+            vr[j] = *(const uint2*)(vb + (size_t)min(b * kKb + kq + 16 * j, last_pos) * row + 8 * dg);
+        if (tid < kKb) vsr = vscales[(size_t)min(b * kKb + tid, last_pos) * n_kv + kvh];
+    };
+    auto store_k = [&](uint32_t f) {
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-            const uint32_t w0 = vr[0][c], w1 = vr[1][c], w2 = vr[2][c], w3 = vr[3][c];
-            const uint32_t a0 = __builtin_amdgcn_perm(w1, w0, 0x05010400u), a1 = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
-            const uint32_t b0 = __builtin_amdgcn_perm(w3, w2, 0x05010400u), b1 = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
-            L.vT[vt_at(16 * dg + 4 * c + 0, kq)] = __builtin_amdgcn_perm(b0, a0, 0x05040100u);
-            L.vT[vt_at(16 * dg + 4 * c + 1, kq)] = __builtin_amdgcn_perm(b0, a0, 0x07060302u);
-            L.vT[vt_at(16 * dg + 4 * c + 2, kq)] = __builtin_amdgcn_perm(b1, a1, 0x05040100u);
-            L.vT[vt_at(16 * dg + 4 * c + 3, kq)] = __builtin_amdgcn_perm(b1, a1, 0x07060302u);
+        for (int j = 0; j < 2; ++j) *(u32x4*)&L.K[f][kk + 32 * j][16 * kc] = kr[j];
+        if (tid < kKb) L.ks[f][tid] = ksr;
+    };
+    auto store_v = [&](uint32_t f) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c) {
+            const uint32_t w0 = c ? vr[0].y : vr[0].x, w1 = c ? vr[1].y : vr[1].x;
+            const uint32_t w2 = c ? vr[2].y : vr[2].x, w3 = c ? vr[3].y : vr[3].x;
+            const uint32_t a0 = __builtin_amdgcn_perm(w1, w0, 0x05010400u);
+            const uint32_t a1 = __builtin_amdgcn_perm(w1, w0, 0x07030602u);
+            const uint32_t b0 = __builtin_amdgcn_perm(w3, w2, 0x05010400u);
+            const uint32_t b1 = __builtin_amdgcn_perm(w3, w2, 0x07030602u);
+            L.vT[f][vt_at(8 * dg + 4 * c + 0, kq)] = __builtin_amdgcn_perm(b0, a0, 0x05040100u);
+            L.vT[f][vt_at(8 * dg + 4 * c + 1, kq)] = __builtin_amdgcn_perm(b0, a0, 0x07060302u);
+            L.vT[f][vt_at(8 * dg + 4 * c + 2, kq)] = __builtin_amdgcn_perm(b1, a1, 0x05040100u);
+            L.vT[f][vt_at(8 * dg + 4 * c + 3, kq)] = __builtin_amdgcn_perm(b1, a1, 0x07060302u);
         }
-        if (tid < kKb) {
-            L.ks[tid] = ksr;
-            L.vs[tid] = vsr;
-        }
+        if (tid < kKb) L.vs[f][tid] = vsr;
     };
 
-    if (kb0 < kb1) load(kb0);
-    // piece slot 3 of every probability row stays zero
-    for (uint32_t i = tid; i < sizeof(L.P) / 4; i += 256) ((uint32_t*)&L.P[0][0][0])[i] = 0u;
-    __syncthreads();  // q pieces and the zero rows complete
-
-    // per owned tile tt (tile 2w + tt): A operand (lane (r, g): piece r%4 of
-    // query row 4i + r/4, dims 64g .. 64g+63; piece slot 3 is zero) and the
-    // lane's query row 4i + g in the D layout with its softmax state
-    u32x4 qa[2][4];
-    uint32_t my_tq[2], my_head[2], my_pos[2];
-    float qs[2][3], m[2], l[2], o[2][16];
-    v4i acc[2][16];  // softmax . V since the last flush, int32 per piece (rows 4*g4 + piece)
-#pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-        const uint32_t i = 2 * w + tt, ar = 4 * i + r16 / 4, pc = r16 % 4;
-#pragma unroll
-        for (int c = 0; c < 4; ++c)
-            qa[tt][c] = pc < kQPieces ? *(const u32x4*)&L.q[ar][pc][64 * g4 + 16 * c] : u32x4{0u, 0u, 0u, 0u};
-        const uint32_t mr = 4 * i + g4;
-        my_tq[tt] = mr / G;
-        my_head[tt] = kvh + n_kv * (mr % G);
-        my_pos[tt] = pos0 + t_first + my_tq[tt];
-#pragma unroll
-        for (int pc2 = 0; pc2 < 3; ++pc2) qs[tt][pc2] = L.qs[mr][pc2];
-        m[tt] = -INFINITY;
-        l[tt] = 0.f;
-#pragma unroll
-        for (int d = 0; d < 16; ++d) {
-            o[tt][d] = 0.f;
-            acc[tt][d] = v4i{0, 0, 0, 0};
-        }
+    if (kb0 < kb1) {
+        load_k(kb0);
+        load_v(kb0);
     }
-    constexpr float scale = 1.0f / 16.0f;  // 1/sqrt(256)
+    // piece slot 3 of every probability row stays zero
+    for (uint32_t i = tid; i < sizeof(L.P) / 4; i += 512) ((uint32_t*)&L.P[0][0][0])[i] = 0u;
     // fixed piece steps for the whole walk: p = e * vs <= vs_max (e <= 1
     // against the row's running maximum m)
-    float vmax;
     {
         float v = 0.0f;
         const uint32_t pend = min(kb1 * kKb, last_pos + 1);
-        for (uint32_t p = kb0 * kKb + tid; p < pend; p += 256) v = fmaxf(v, vscales[(size_t)p * n_kv + kvh]);
+        for (uint32_t p = kb0 * kKb + tid; p < pend; p += 512) v = fmaxf(v, vscales[(size_t)p * n_kv + kvh]);
         v = wave_max(v);
         if (lane == 0) L.vsw[w] = v;
-        __syncthreads();
-        vmax = fmaxf(fmaxf(L.vsw[0], L.vsw[1]), fmaxf(L.vsw[2], L.vsw[3]));
     }
+    if (kb0 < kb1) {
+        store_k(0);
+        store_v(0);
+        load_k(min(kb0 + 1, kb1 - 1));
+        load_v(min(kb0 + 1, kb1 - 1));
+    }
+    __syncthreads();  // q pieces, the zero rows, the maxima and the first block complete
+
+    // A operand (lane (r, g): piece r%4 of query row 4w + r/4, dims 64g ..
+    // 64g+63; piece slot 3 is zero) and the lane's query row 4w + g in the D
+    // layout with its softmax state
+    v4i qa[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+        qa[c] = r16 % 4 < kQPieces ? *(const v4i*)&L.q[4 * w + r16 / 4][r16 % 4][64 * g4 + 16 * c] : v4i{0, 0, 0, 0};
+    const uint32_t mr = 4 * w + g4, my_tq = mr / G, my_head = kvh + n_kv * (mr % G), my_pos = pos0 + t_first + my_tq;
+    const float qs0 = L.qs[mr][0], qs1 = L.qs[mr][1], qs2 = L.qs[mr][2];
+    float m = -INFINITY, l = 0.f, o[16];
+    v4i acc[16];  // softmax . V since the last flush, int32 per piece (rows 4*g4 + piece)
+#pragma unroll
+    for (int d = 0; d < 16; ++d) {
+        o[d] = 0.f;
+        acc[d] = v4i{0, 0, 0, 0};
+    }
+    constexpr float scale = 1.0f / 16.0f;  // 1/sqrt(256)
+    float vmax = L.vsw[0];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) vmax = fmaxf(vmax, L.vsw[i]);
     const float st0 = vmax > 0.0f ? vmax * (1.0f / 127.0f) : 1.0f, iv0 = vmax > 0.0f ? 127.0f / vmax : 1.0f;
     const float st1 = st0 * (1.0f / 254.0f), iv1 = iv0 * 254.0f;
     const float st2 = st1 * (1.0f / 254.0f), iv2 = iv1 * 254.0f;
+    // The score products start at the bit pattern of 1.5 * 2^23, so that a sum
+    // read as a float less that is the sum (|sum| <= 256 * 127 * 128 < 2^22):
+    // a subtraction where a conversion issues at half the rate.
+    const v4i magic = {0x4B400000, 0x4B400000, 0x4B400000, 0x4B400000};
+    auto value = [](int c) { return __int_as_float(c) - 12582912.0f; };
 
-    for (uint32_t b = kb0; b < kb1; ++b) {
-        __syncthreads();  // the previous block's readers of K, vT are done
-        store();
-        __syncthreads();
-        if (b + 1 < kb1) load(b + 1);
-        // ---- scores of both owned tiles: 4 key tiles x 8 k-steps each; K
-        // operand lane (r, g) = position 16kt + r, dims 64g .. 64g+63
-        // (one key tile's K operand at a time: 16 VGPRs instead of 64)
-        v4i C[2][4];
+    // ---- scores: 4 key tiles x 4 k-steps; K operand lane (r, g) = position
+    // 16kt + r, dims 64g .. 64g+63
+    v4i C[4];
+    float sc[4], bm;
+    auto products = [&](uint32_t f) {
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) {
-            u32x4 kb[4];
+            C[kt] = magic;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) kb[c] = *(const u32x4*)&L.K[16 * kt + r16][64 * g4 + 16 * c];
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                C[tt][kt] = v4i{0, 0, 0, 0};
-#pragma unroll
-                for (int m8 = 0; m8 < 8; ++m8) {
-                    const u32x4 a = qa[tt][m8 / 2], bb = kb[m8 / 2];
-                    const long A = (m8 & 1) ? pack2(a.z, a.w) : pack2(a.x, a.y);
-                    const long B = (m8 & 1) ? pack2(bb.z, bb.w) : pack2(bb.x, bb.y);
-                    C[tt][kt] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A, B, C[tt][kt], 0, 0, 0);
-                }
-            }
+            for (int c = 0; c < 4; ++c)
+                C[kt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                    qa[c], *(const v4i*)&L.K[f][16 * kt + r16][64 * g4 + 16 * c], C[kt], 0, 0, 0);
         }
+    };
+    auto scores = [&](uint32_t b, uint32_t f) {  // of the products of block b, and whether a maximum rises
+        bm = -INFINITY;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) {
+            const uint32_t kp = b * kKb + 16 * kt + r16;
+            const float raw = (qs0 * value(C[kt][0]) + qs1 * value(C[kt][1])) + qs2 * value(C[kt][2]);
+            sc[kt] = kp <= my_pos ? raw * L.ks[f][16 * kt + r16] * scale : -INFINITY;
+            bm = fmaxf(bm, sc[kt]);
+        }
+        bm = row16_max(bm);
+        const bool rises = __any(bm > m);
+        if (lane == 0) L.rise[f][w] = rises;
+    };
+    if (kb0 < kb1) {
+        products(0);
+        scores(kb0, 0);
+        store_k(1);
+        load_k(min(kb0 + 2, kb1 - 1));
+    }
+    __syncthreads();
+
+    for (uint32_t b = kb0; b < kb1; ++b) {
+        // In LDS: V of block b, K of block b + 1.  K of block b and V of block
+        // b - 1 are read: their buffers take K of b + 2 and V of b + 1.  (Past
+        // the walk's end the last block again, its scores unused.)
+        const uint32_t f = (b - kb0) & 1;
+        products(f ^ 1);
+        store_k(f);
+        store_v(f ^ 1);
+        load_k(min(b + 3, kb1 - 1));
+        load_v(min(b + 2, kb1 - 1));
         // ---- softmax against the running row maximum m; lane (r16 = position
-        // in key tile, g4 = query row).  When a row's maximum rises (or every
-        // kFlushBlocks blocks, the int32 bound) the wave flushes: o = (o +
-        // sum_j step_j * acc_j) * exp(m_old - m_new), acc = 0, l rescaled.
-        // Otherwise probabilities keep the fixed steps and softmax . V
-        // accumulates in the MFMA's int32 registers with no fp32 epilogue.
-        float sc[2][4], bm[2];
+        // in key tile, g4 = query row).  When a maximum of the pair's rows
+        // rises (or every kFlushBlocks blocks, the int32 bound) the wave
+        // flushes: o = (o + sum_j step_j * acc_j) * exp(m_old - m_new), acc =
+        // 0, l rescaled.  Otherwise probabilities keep the fixed steps and
+        // softmax . V accumulates in the MFMA's int32 registers with no fp32
+        // epilogue.
+        if ((L.rise[f][w] | L.rise[f][w ^ 1]) || ((b - kb0) % kFlushBlocks == 0 && b > kb0)) {
+            // -inf until a row sees a visible position (a later segment
+            // may start past a row's own position)
+            const float mn = fmaxf(m, bm);
+            const float corr = mn == -INFINITY ? 1.0f : __expf(m - mn);  // first: exp(-inf) = 0
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            bm[tt] = -INFINITY;
-#pragma unroll
-            for (int kt = 0; kt < 4; ++kt) {
-                const uint32_t kp = b * kKb + 16 * kt + r16;
-                const v4i c4 = C[tt][kt];
-                const float raw = (qs[tt][0] * (float)c4[0] + qs[tt][1] * (float)c4[1]) + qs[tt][2] * (float)c4[2];
-                sc[tt][kt] = kp <= my_pos[tt] ? raw * L.ks[16 * kt + r16] * scale : -INFINITY;
-                bm[tt] = fmaxf(bm[tt], sc[tt][kt]);
+            for (int dt = 0; dt < 16; ++dt) {
+                const v4i c = acc[dt];
+                o[dt] = (o[dt] + ((st0 * (float)c[0] + st1 * (float)c[1]) + st2 * (float)c[2])) * corr;
+                acc[dt] = v4i{0, 0, 0, 0};
             }
-            bm[tt] = row16_max(bm[tt]);
-        }
-        if (__any(bm[0] > m[0] || bm[1] > m[1]) || ((b - kb0) % kFlushBlocks == 0 && b > kb0)) {
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                // -inf until a row sees a visible position (a later segment
-                // may start past a row's own position)
-                const float mn = fmaxf(m[tt], bm[tt]);
-                const float corr = mn == -INFINITY ? 1.0f : __expf(m[tt] - mn);  // first: exp(-inf) = 0
-#pragma unroll
-                for (int dt = 0; dt < 16; ++dt) {
-                    const v4i c = acc[tt][dt];
-                    o[tt][dt] = (o[tt][dt] + ((st0 * (float)c[0] + st1 * (float)c[1]) + st2 * (float)c[2])) * corr;
-                    acc[tt][dt] = v4i{0, 0, 0, 0};
-                }
-                l[tt] *= corr;
-                m[tt] = mn;
-            }
+            l *= corr;
+            m = mn;
         }
         // probability x V row scale as three int8 pieces (fixed steps): row
-        // 4*g4 + piece of tile i; the four key tiles' values of position r16
+        // 4*g4 + piece of the tile; the four key tiles' values of position r16
         // are bytes 0..3 of dword r16 (contraction index 4*r16 + kt)
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const uint32_t i = 2 * w + tt;
-            const float mu = m[tt] == -INFINITY ? 0.0f : m[tt];  // every score masked while m is -inf
+        {
+            const float mu = m == -INFINITY ? 0.0f : m;  // every score masked while m is -inf
             uint32_t pw[kQPieces] = {0u, 0u, 0u};
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt) {
-                const float e = __expf(sc[tt][kt] - mu);  // <= 1; masked: 0
-                l[tt] += e;
-                const float pr = e * L.vs[16 * kt + r16];
+                const float e = __expf(sc[kt] - mu);  // <= 1; masked: 0
+                l += e;
+                const float pr = e * L.vs[f][16 * kt + r16];
                 const float q0 = fminf(rintf(pr * iv0), 127.0f);
                 const float r1 = fmaf(-q0, st0, pr);
                 const float q1 = fminf(fmaxf(rintf(r1 * iv1), -127.0f), 127.0f);
@@ -320,55 +329,46 @@ __global__ __launch_bounds__(256) void k_attn_prefill(const float* __restrict__ 
                 pw[2] |= (uint32_t)(uint8_t)(int8_t)q2 << (8 * kt);
             }
 #pragma unroll
-            for (uint32_t pc = 0; pc < kQPieces; ++pc) ((uint32_t*)&L.P[i][4 * g4 + pc][0])[r16] = pw[pc];
+            for (uint32_t pc = 0; pc < kQPieces; ++pc) ((uint32_t*)&L.P[w][4 * g4 + pc][0])[r16] = pw[pc];
         }
+        scores(b + 1, f ^ 1);
         __builtin_amdgcn_s_waitcnt(0xc07f);  // this wave's P dwords are in LDS before its reads below
         __builtin_amdgcn_wave_barrier();
-        // ---- P . V: 16 dim tiles x 2 k-steps per tile (lane group g4:
-        // contraction indices 16g4 .. 16g4+15); each V operand serves both tiles
-        long A[2][2];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            const uint2* ap = (const uint2*)&L.P[2 * w + tt][r16][16 * g4];
-            const uint2 a0 = ap[0], a1 = ap[1];
-            A[tt][0] = pack2(a0.x, a0.y);
-            A[tt][1] = pack2(a1.x, a1.y);
-        }
+        // ---- P . V: 16 dim tiles, one step of 64 positions each (lane group
+        // g4: contraction indices 16g4 .. 16g4+15)
+        const uint2* ap = (const uint2*)&L.P[w][r16][16 * g4];
+        const uint2 a0 = ap[0], a1 = ap[1];
+        const v4i A = {(int)a0.x, (int)a0.y, (int)a1.x, (int)a1.y};
 #pragma unroll
         for (int dt = 0; dt < 16; ++dt) {
-            const uint2* bp = (const uint2*)&L.vT[vt_at(16 * dt + r16, 4 * g4)];
+            const uint2* bp = (const uint2*)&L.vT[f][vt_at(16 * dt + r16, 4 * g4)];
             const uint2 b0 = bp[0], b1 = bp[1];
-#pragma unroll
-            for (int tt = 0; tt < 2; ++tt) {
-                acc[tt][dt] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[tt][0], pack2(b0.x, b0.y), acc[tt][dt], 0, 0, 0);
-                acc[tt][dt] = __builtin_amdgcn_mfma_i32_16x16x32_i8(A[tt][1], pack2(b1.x, b1.y), acc[tt][dt], 0, 0, 0);
-            }
+            acc[dt] = __builtin_amdgcn_mfma_i32_16x16x64_i8(A, v4i{(int)b0.x, (int)b0.y, (int)b1.x, (int)b1.y}, acc[dt],
+                                                            0, 0, 0);
         }
+        __syncthreads();
     }
+    const float lt = row16_sum(l);
+    if (my_tq >= n_tok) return;
+    const size_t qi = (size_t)(t_first + my_tq) * n_heads + my_head;
+    if (S == 1) {  // the whole walk: normalized output
+        const float inv = 1.0f / lt;
+        float* dst = out + qi * kHd;
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt) {
-        const float lt = row16_sum(l[tt]);
-        if (my_tq[tt] >= n_tok) continue;
-        const size_t qi = (size_t)(t_first + my_tq[tt]) * n_heads + my_head[tt];
-        if (S == 1) {  // the whole walk: normalized output
-            const float inv = 1.0f / lt;
-            float* dst = out + qi * kHd;
+        for (int dt = 0; dt < 16; ++dt) {
+            const v4i c = acc[dt];
+            dst[16 * dt + r16] = (o[dt] + ((st0 * (float)c[0] + st1 * (float)c[1]) + st2 * (float)c[2])) * inv;
+        }
+    } else {  // segment partial: unnormalized o, row maximum, row sum
+        float* dst = part + ((size_t)seg * T * n_heads + qi) * kPartStride;
 #pragma unroll
-            for (int dt = 0; dt < 16; ++dt) {
-                const v4i c = acc[tt][dt];
-                dst[16 * dt + r16] = (o[tt][dt] + ((st0 * (float)c[0] + st1 * (float)c[1]) + st2 * (float)c[2])) * inv;
-            }
-        } else {  // segment partial: unnormalized o, row maximum, row sum
-            float* dst = part + ((size_t)seg * T * n_heads + qi) * kPartStride;
-#pragma unroll
-            for (int dt = 0; dt < 16; ++dt) {
-                const v4i c = acc[tt][dt];
-                dst[16 * dt + r16] = o[tt][dt] + ((st0 * (float)c[0] + st1 * (float)c[1]) + st2 * (float)c[2]);
-            }
-            if (r16 == 0) {
-                dst[kHd] = m[tt];
-                dst[kHd + 1] = lt;
-            }
+        for (int dt = 0; dt < 16; ++dt) {
+            const v4i c = acc[dt];
+            dst[16 * dt + r16] = o[dt] + ((st0 * (float)c[0] + st1 * (float)c[1]) + st2 * (float)c[2]);
+        }
+        if (r16 == 0) {
+            dst[kHd] = m;
+            dst[kHd + 1] = lt;
         }
     }
 }
@@ -427,15 +427,15 @@ extern "C" int ec_attn_prefill(const float* q, const int8_t* keys, const int8_t*
     float* part = (float*)ws;
     switch (G) {
         case 1:
-            hipLaunchKernelGGL(k_attn_prefill<1>, grid, dim3(256), 0, st, q, keys, vals, kscales, vscales, out, part, T,
+            hipLaunchKernelGGL(k_attn_prefill<1>, grid, dim3(512), 0, st, q, keys, vals, kscales, vscales, out, part, T,
                                (uint32_t)pos0, n_kv, S);
             break;
         case 2:
-            hipLaunchKernelGGL(k_attn_prefill<2>, grid, dim3(256), 0, st, q, keys, vals, kscales, vscales, out, part, T,
+            hipLaunchKernelGGL(k_attn_prefill<2>, grid, dim3(512), 0, st, q, keys, vals, kscales, vscales, out, part, T,
                                (uint32_t)pos0, n_kv, S);
             break;
         case 4:
-            hipLaunchKernelGGL(k_attn_prefill<4>, grid, dim3(256), 0, st, q, keys, vals, kscales, vscales, out, part, T,
+            hipLaunchKernelGGL(k_attn_prefill<4>, grid, dim3(512), 0, st, q, keys, vals, kscales, vscales, out, part, T,
                                (uint32_t)pos0, n_kv, S);
             break;
         default:

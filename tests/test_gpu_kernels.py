@@ -351,6 +351,31 @@ def test_attention_prefill(hip, oc, T, pos0, n_heads, n_kv):
         print(f"T {T} pos0 {pos0} ({tag}, workspace {nws} B): worst per-token rel_l2 {worst:.2e}")
 
 
+@pytest.mark.parametrize("T,pos0", [(1, 62), (1, 63), (1, 64), (2, 127), (40, 100), (33, 191), (9, 1030)])
+@pytest.mark.parametrize("n_heads,n_kv", [(16, 4), (8, 4), (4, 4)])
+def test_attention_prefill_short_walks(hip, oc, T, pos0, n_heads, n_kv):
+    """Walks of one to four key blocks (K and V alternate between two buffers, the last block's successors are not
+    there) and segments of one or two, with the largest score products there are: equal |q| and keys of -128 or 127
+    sum to 256 * 127 * 128 in the first piece.  Against the oracle per token, 1e-5 as above."""
+    import torch
+    hd, ctx = 256, pos0 + T
+    keys, vals, ks, vs, _, _ = _kv_case(oc, 1, [ctx], ctx, n_kv, hd, 17 + T)
+    keys[0, ::3] = -128
+    keys[0, 1::5] = 127
+    q = synth.activations(18 + pos0, T * n_heads * hd).reshape(T, n_heads * hd)
+    q[::2] = 0.01
+    q[1::4] = -0.01
+    ws = empty(max(hip.attn_prefill_ws_bytes(T, n_heads, ctx), 16), torch.uint8)
+    for w in (ws, None):
+        out = dev(np.full(T * n_heads * hd, 7.0, np.float32))
+        hip.attn_prefill(dev(q), dev(keys[0]), dev(vals[0]), dev(ks[0]), dev(vs[0]), out, T, pos0, n_heads, n_kv, hd,
+                         ctx, ws=w)
+        got = host(out).reshape(T, n_heads * hd)
+        for t in range(T):
+            ref = oc.attn_decode(q[t], keys[0], vals[0], ks[0], vs[0], n_heads, n_kv, hd, pos0 + t + 1)
+            assert rel_l2(got[t], ref) < 1e-5, (w is None, t)
+
+
 def _pack_q_pieces(q, n_heads, n_kv):
     """q [n_seq][n_heads*256] -> the three-piece int8 A-operand layout of
     ec_attn_decode_packed: per (seq, kv head) [3G rows][4 k-groups][64 bytes],
