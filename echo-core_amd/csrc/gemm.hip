@@ -50,9 +50,9 @@
 // M x N x K, us, this kernel / the one before it (64 x 64 workgroup tiles,
 // 16x16x32 MFMA, conversion + product + FMA per element, scales through a
 // workgroup-wide LDS stage with a barrier per chunk; same bits for Q8_0):
-//   Q8_0 1024x18432x2560 157 / 211, 1024x2560x9216 106 / 125, 512x12352x2560
-//        69 / 79, 512x2560x9216 62 / 75, 200x2560x9216 43 / 57,
-//        130x12352x2560 28 / 37, 40x18432x2560 20 / 23, 40x2560x9216 19 / 56
+//   Q8_0 1024x18432x2560 160 / 203, 1024x2560x9216 91 / 121, 512x12352x2560
+//        69 / 78, 512x2560x9216 59 / 75, 200x2560x9216 44 / 57,
+//        130x12352x2560 24 / 37, 40x18432x2560 20 / 23, 40x2560x9216 19 / 56
 //   Q4_K 1024x18432x2560 175 / 270, 387x18432x2560 76 / 121, 387x2560x9216
 //        50 / 88, 40x2560x9216 17 / 56
 // Also tried at Q8_0 1024x18432x2560: both operands staged in LDS by the
@@ -60,7 +60,8 @@
 // token scales spread over the lanes by v_mfma_f32_16x16x4_f32 instead of LDS
 // reads (157 with two operations), 64 x 64 tiles per wave (171), two tiles'
 // products in flight at two waves per SIMD (171), a barrier per chunk to keep
-// the four waves on the same lines of L1 (no change).
+// four waves on the same lines of L1 (no change), operands three halves of a
+// chunk ahead instead of one (no change here nor at 130 tokens).
 #include <type_traits>
 
 #include "gemm_act.hpp"
@@ -192,30 +193,30 @@ __device__ __forceinline__ void static_for(F&& f) {
 // them back as float4s that all lanes of a half share; only its own lanes
 // read them, and a wave's LDS accesses stay in order.
 //
-// Workgroups of four waves: KW = 1, 2 x 2 tiles with all of K each; KW = 4, one
-// tile, a quarter of K each.  ONEC: one result tile in flight (a second one's
-// 16 registers would cost a wave per SIMD, or spill).
+// A workgroup is one tile: KW = 1, one wave with all of K (2 x 2 waves of
+// neighbouring tiles ran 1024x2560x9216 in 104 us instead of 91 and
+// 130x18432x2560 in 41 instead of 35: waves that end early leave their place
+// to the next at once); KW = 4, four waves with a quarter of K each.  ONEC:
+// one result tile in flight (a second one's 16 registers would cost a wave
+// per SIMD, or spill).
 template <int FMT, int TT, int RT, int KW, int MINW, bool ONEC>
-__global__ __launch_bounds__(256, MINW) void k_gemm(const uint8_t* __restrict__ W, const uint8_t* __restrict__ xt,
+__global__ __launch_bounds__(64 * KW, MINW) void k_gemm(const uint8_t* __restrict__ W, const uint8_t* __restrict__ xt,
                                                     float* __restrict__ y, uint32_t M, uint32_t N, uint32_t n_tt,
                                                     uint32_t n_rt, uint32_t nG, uint32_t nbp, size_t xd_off,
                                                     size_t dxs_off, uint32_t ldy, int accumulate, uint32_t gx,
                                                     uint32_t gy) {
     constexpr bool Q4 = FMT == EC_Q4_K;
-    constexpr int TW = KW == 1 ? 2 : 1, RW = TW;      // waves over token and row tiles
     constexpr int NX = Q4 ? 8 : 4, E = TT * RT * 16;  // scale rows per token in LDS; sums per lane
-    constexpr size_t kScale = 4 * 2 * NX * 32 * TT * sizeof(float), kSums = KW == 1 ? 0 : KW * E * 64 * sizeof(float);
+    constexpr size_t kScale = KW * 2 * NX * 32 * TT * sizeof(float), kSums = KW == 1 ? 0 : KW * E * 64 * sizeof(float);
     __shared__ __align__(16) uint8_t lds[kScale > kSums ? kScale : kSums];
     // consecutive workgroups run on consecutive XCDs: an XCD takes every eighth
     // row block and all of its token blocks, so its L2 reads those weights once
     const uint32_t id = blockIdx.x, kk = id >> 3, bx = (kk / gy) * 8 + (id & 7), by = kk % gy;
     if (bx >= gx) return;
     const uint32_t lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), h = lane >> 5;
-    const uint32_t T0 = 2 * TT * (KW == 1 ? by * TW + w % TW : by);  // first 16-token tile
-    const uint32_t R0 = 2 * RT * (KW == 1 ? bx * RW + w / TW : bx);  // first 16-row tile
-    if (KW == 1 && (T0 >= n_tt || R0 >= n_rt)) return;
-    const uint32_t G0 = KW == 1 ? 0 : w * nG / KW, G1 = KW == 1 ? nG : (w + 1) * nG / KW;  // chunks of 4 blocks
-    float(*sc_s)[NX][32 * TT] = (float(*)[NX][32 * TT])(lds + w * (kScale / 4));  // this wave's [buffer][row][token]
+    const uint32_t T0 = 2 * TT * by, R0 = 2 * RT * bx;        // first 16-token and 16-row tile
+    const uint32_t G0 = w * nG / KW, G1 = (w + 1) * nG / KW;  // this wave's chunks of 4 blocks
+    float(*sc_s)[NX][32 * TT] = (float(*)[NX][32 * TT])(lds + w * (kScale / KW));  // this wave's [buffer][row][token]
 
     // operand lane l: row l % 32 of the 32-row tile, K groups h and h + 2 (8 elements each) of every block.
     // Wave-uniform bases and 32-bit lane offsets within the tile.
@@ -546,11 +547,10 @@ __global__ __launch_bounds__(64, 2) void k_gemm_q8_16(const uint8_t* __restrict_
 template <int FMT, int TT, int RT, int KW, int MINW, bool ONEC>
 static void launch_tile(const XtLayout& L, const uint8_t* W, const uint8_t* xt, float* y, uint32_t M, uint32_t N,
                         uint32_t ldy, int accumulate, hipStream_t st) {
-    constexpr uint32_t nt = 2 * TT * (KW == 1 ? 2 : 1), nr = 2 * RT * (KW == 1 ? 2 : 1);  // 16-wide tiles per workgroup
     const uint32_t n_tt = L.Mp / 16, n_rt = round_up(N, 16) / 16;
-    const uint32_t gx = (n_rt + nr - 1) / nr, gy = (n_tt + nt - 1) / nt;
-    hipLaunchKernelGGL((k_gemm<FMT, TT, RT, KW, MINW, ONEC>), dim3(round_up(gx, 8) * gy), dim3(256), 0, st, W, xt, y, M,
-                       N, n_tt, n_rt, L.Kp / 128, L.Kp / 32, L.xd_off, L.dxs_off, ldy, accumulate, gx, gy);
+    const uint32_t gx = (n_rt + 2 * RT - 1) / (2 * RT), gy = (n_tt + 2 * TT - 1) / (2 * TT);
+    hipLaunchKernelGGL((k_gemm<FMT, TT, RT, KW, MINW, ONEC>), dim3(round_up(gx, 8) * gy), dim3(64 * KW), 0, st, W, xt, y,
+                       M, N, n_tt, n_rt, L.Kp / 128, L.Kp / 32, L.xd_off, L.dxs_off, ldy, accumulate, gx, gy);
 }
 
 template <int RT, int D>
@@ -562,16 +562,16 @@ static void launch_q8_16(const XtLayout& L, const uint8_t* W, const uint8_t* xt,
 }
 
 // The tile, by the number of 32 x 32 tiles for 1024 SIMDs.  32 x 64 per wave
-// reads less per product and needs a few waves per SIMD (18432 tiles:
-// 1024x18432 157 us, 188 with 32 x 32; 9216: 512x18432 82 / 90; 6176:
-// 512x12352 70 / 69; 4032: 200x18432 49 / 45).  32 x 32 until a SIMD has less
-// than about 1.2 waves (1280: 512x2560x9216 62, 84 with 16 x 32; 1152:
-// 40x18432 21 / 20; 560: 200x2560x9216 55 / 43), then 16 x 32 down to half a
-// wave (720 waves: 130x2560x4096 16, 18 with 16 x 16; 240: 40x2560x9216 30 / 19).
+// reads less per product and needs two waves per SIMD (18432 tiles:
+// 1024x18432 160 us, 198 with 32 x 32; 6144: 1024x6144 55 / 62; 4032:
+// 200x18432 40 / 48; 3072: 512x6144 36 / 32).  32 x 32 until a SIMD has less
+// than about 1.2 waves (1280: 512x2560x9216 59, 84 with 16 x 32; 1152:
+// 40x18432 21 / 20; 800: 300x2560x9216 55 / 51), then 16 x 32 down to half a
+// wave (720 waves: 130x2560x4096 17, 18 with 16 x 16; 240: 40x2560x9216 30 / 19).
 static void launch_q8(const XtLayout& L, const uint8_t* W, const uint8_t* xt, float* y, uint32_t M, uint32_t N,
                       uint32_t ldy, int accumulate, hipStream_t st) {
     const uint64_t tiles = (uint64_t)((M + 31) / 32) * ((N + 31) / 32);
-    if (tiles >= 8192)
+    if (tiles >= 4000)
         launch_tile<EC_Q8_0, 1, 2, 1, 3, true>(L, W, xt, y, M, N, ldy, accumulate, st);
     else if (tiles >= 1216)
         launch_tile<EC_Q8_0, 1, 1, 1, 3, true>(L, W, xt, y, M, N, ldy, accumulate, st);

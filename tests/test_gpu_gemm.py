@@ -115,12 +115,12 @@ def test_gemm(hip, oc, fmt, M, N, K):
 
 
 # Edges of the 16-, 32- and 64-wide tiles, one chunk to a few per wave (Q4_K: empty K quarters at K = 256), and
-# M x N on both sides of where the tile changes: Q8_0 at 512 tiles of 16 x 32, 1216 and 8192 of 32 x 32; Q4_K at 768
+# M x N on both sides of where the tile changes: Q8_0 at 512 tiles of 16 x 32, 1216 and 4000 of 32 x 32; Q4_K at 768
 # tiles of 32 x 64 and 1280 of 64 x 64 whose tokens fill them.
 EDGES = [(m, n, k) for m, n in ((1, 7), (16, 33), (17, 16), (31, 65), (33, 31), (64, 64), (65, 17))
          for k in (256, 512, 1280)]
 EDGES += [(m, n, 256) for m, n in ((16, 16384 - 33), (16, 16384 - 31), (33, 608 * 32 - 33), (33, 608 * 32 - 31),
-                                   (100, 65536 - 33), (100, 65536 - 31), (32, 49152 - 65), (32, 49152 - 63),
+                                   (100, 32000 - 33), (100, 32000 - 31), (32, 49152 - 65), (32, 49152 - 63),
                                    (64, 81920 - 65), (64, 81920 - 63), (80, 41000), (352, 12352))]
 
 
