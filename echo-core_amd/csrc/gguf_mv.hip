@@ -79,6 +79,9 @@ __device__ __forceinline__ void row_sums_store(const float* red, uint32_t ncol, 
     if (t == G0 && rr < nr) y[r0 + rr] = yp + acc;
 }
 
+// The walking kernel (below, for many rows).  kWalkThreads bounds its
+// workgroups so that x's 64 values and a row in flight fit in registers.
+constexpr uint32_t kWalkThreads = 640;
 // Block-pair form (K % 64 == 0): thread column c owns blocks 2c and 2c + 1
 // of its rows, 68 bytes at a dword-aligned offset (the row stride nb * 34 is
 // a multiple of 4), loaded straight from memory as four 16-byte loads and a
@@ -229,6 +232,28 @@ __device__ __forceinline__ void q4_scale_min(uint32_t w0, uint32_t w1, uint32_t 
     mn1 = hi ? ((c >> 12) & 15u) | ((b >> 10) & 48u) : (b >> 8) & 63u;
 }
 
+// A quarter's share of its row: header h, nibble bytes a (0-15) and b (16-31),
+// x in the reference's position order, xm the sums of x's two pairs.
+__device__ __forceinline__ float q4_quarter(const uint4& h, const uint4& a, const uint4& b, uint32_t g,
+                                            const float (&xv)[64], float2 xm) {
+    uint32_t sc0, mn0, sc1, mn1;
+    q4_scale_min(h.y, h.z, h.w, g, sc0, mn0, sc1, mn1);
+    const float d = h2f(h.x & 0xFFFF), dmin = h2f(h.x >> 16);
+    const uint32_t qw[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    float S[2] = {0.0f, 0.0f};
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {  // bytes 0-15: pair 0, bytes 16-31: pair 1
+        uint32_t lo = qw[k] & 0x0F0F0F0Fu, hi = (qw[k] >> 4) & 0x0F0F0F0Fu;
+        hide_bits(lo), hide_bits(hi);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            S[k / 4] = fmaf((float)((lo >> (8 * e)) & 0xFF), xv[4 * k + e], S[k / 4]);
+            S[k / 4] = fmaf((float)((hi >> (8 * e)) & 0xFF), xv[32 + 4 * k + e], S[k / 4]);
+        }
+    }
+    return ((d * (float)sc0) * S[0] + (d * (float)sc1) * S[1]) - dmin * ((float)mn0 * xm.x + (float)mn1 * xm.y);
+}
+
 // nq_magic = ceil(2^32 / nq): t / nq == umulhi(t, nq_magic) exactly for
 // t, nq < 2^10 (the rounding error t * (nq_magic - 2^32/nq) / 2^32 < 2^-22
 // is below the 1/nq gap to the next integer).
@@ -291,37 +316,118 @@ __global__ __launch_bounds__(q4_f32_max_threads<RPT>()) void k_gguf_q4_K_f32(
         // bytes, and its value is never read -- a branch here would let the
         // compiler sink the weights' loads below the barrier
         const uint32_t rr = ph + i * P;
-        uint32_t sc0, mn0, sc1, mn1;
-        q4_scale_min(hd[i].y, hd[i].z, hd[i].w, g, sc0, mn0, sc1, mn1);
-        const float d = h2f(hd[i].x & 0xFFFF), dmin = h2f(hd[i].x >> 16);
-        const uint32_t qw[8] = {q0[i].x, q0[i].y, q0[i].z, q0[i].w, q1[i].x, q1[i].y, q1[i].z, q1[i].w};
-        float S0 = 0.0f, S1 = 0.0f;
-#pragma unroll
-        for (int k = 0; k < 4; ++k) {  // bytes 0-15: pair 0
-            uint32_t lo = qw[k] & 0x0F0F0F0Fu, hi = (qw[k] >> 4) & 0x0F0F0F0Fu;
-            hide_bits(lo), hide_bits(hi);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                S0 = fmaf((float)((lo >> (8 * e)) & 0xFF), xv[4 * k + e], S0);
-                S0 = fmaf((float)((hi >> (8 * e)) & 0xFF), xv[32 + 4 * k + e], S0);
-            }
-        }
-#pragma unroll
-        for (int k = 4; k < 8; ++k) {  // bytes 16-31: pair 1
-            uint32_t lo = qw[k] & 0x0F0F0F0Fu, hi = (qw[k] >> 4) & 0x0F0F0F0Fu;
-            hide_bits(lo), hide_bits(hi);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                S1 = fmaf((float)((lo >> (8 * e)) & 0xFF), xv[4 * k + e], S1);
-                S1 = fmaf((float)((hi >> (8 * e)) & 0xFF), xv[32 + 4 * k + e], S1);
-            }
-        }
-        const float val = ((d * (float)sc0) * S0 + (d * (float)sc1) * S1) -
-                          dmin * ((float)mn0 * xm.x + (float)mn1 * xm.y);
-        red[ph0 < P ? rr * nq + q : R * nq] = val;  // padding threads: the spare slot
+        red[ph0 < P ? rr * nq + q : R * nq] = q4_quarter(hd[i], q0[i], q1[i], g, xv, xm);  // padding: the spare slot
     }
     __syncthreads();
     row_sums_store(red, nq, nr, G, yp, y, r0);
+}
+
+// Many rows: the workgroups that fit the GPU walk the tiles of P rows (one per
+// thread) blockIdx, blockIdx + gridDim, ... with x staged once and kept in
+// registers, where the kernel above stages it for every tile (151936 x 2560:
+// 190 MB of x from L2 beside 219 MB of weights).  The next tile's loads are
+// issued when this tile's are used up (a row past the last reads the last one
+// again); the quarter values alternate between two LDS areas, one barrier per
+// tile; rows' sums as above, G lanes each, in the same order: the same bits.
+// P is what fills four whole waves: with the five of the kernel above (2560
+// columns) a CU held two workgroups.  us, this / the kernel above: 151936 x
+// 2560 59 / 64, 65536 x 2560 22 / 28, 32768 x 2560 13.4 / 15.8, 50000 x 4096
+// 26.5 / 35, 20000 x 9216 31 / 37.5; two to four rows in flight per thread were
+// slower (60-70 at 151936 x 2560).  What is left is arithmetic: a conversion
+// (half rate) and an FMA per weight beside the unpacking, about half the time.
+template <int XPT, int G>
+__global__ __launch_bounds__(kWalkThreads) void k_gguf_q4_K_f32_walk(const uint8_t* __restrict__ W,
+                                                                     const float* __restrict__ x, float* __restrict__ y,
+                                                                     uint32_t M, uint32_t nsb, uint32_t P,
+                                                                     uint32_t nq_magic) {
+    extern __shared__ uint8_t lds[];
+    const uint32_t t = threadIdx.x, T = blockDim.x, nq = 4 * nsb;
+    float* xs = (float*)lds;
+    float2* xsum = (float2*)(xs + (size_t)nq * kQ4XStride);
+    float* rd = (float*)(xsum + nq);  // 2 x ([P][nq] + 1)
+    float* other = rd + P * nq + 1;
+    const uint32_t ph0 = __umulhi(t, nq_magic), q = t - ph0 * nq;
+    const uint32_t ph = min(ph0, P - 1), sb = q / 4, g = q % 4;  // padding threads: q < nq, ph0 >= P
+    const size_t rowbytes = (size_t)nsb * 144;
+    const uint32_t n4 = 16 * nq, tiles = (M + P - 1) / P;
+    float4 xf[XPT];  // float4s t, t + T, ... of x
+#pragma unroll
+    for (int j = 0; j < XPT; ++j) xf[j] = ((const float4*)x)[min(t + j * T, n4 - 1)];
+    __builtin_amdgcn_sched_barrier(0);  // keep x's loads ahead of the weights'
+    uint4 hd, q0, q1;
+    float yp;  // the previous y of row t / G of the tile
+    auto load = [&](uint32_t tile) {
+        const uint8_t* bp = W + (size_t)min(tile * P + ph, M - 1) * rowbytes + 144 * (size_t)sb;
+        hd = *(const uint4*)bp;
+        q0 = ld_nt16(bp + 16 + 32 * g);
+        q1 = ld_nt16(bp + 32 + 32 * g);
+    };
+    auto load_y = [&](uint32_t tile) { yp = y[min(tile * P + t / G, M - 1)]; };
+    load(blockIdx.x);
+    load_y(blockIdx.x);
+#pragma unroll
+    for (int j = 0; j < XPT; ++j) {
+        const uint32_t c4 = t + j * T;
+        const uint32_t o = c4 < n4 ? (c4 / 16) * kQ4XStride + 4 * (c4 % 16) : (nq - 1) * kQ4XStride + 64;
+        *(float4*)(xs + o) = xf[j];
+        float ps = (xf[j].x + xf[j].y) + (xf[j].z + xf[j].w);
+        ps += lane_xor<1>(ps);
+        ps += lane_xor<2>(ps);
+        ps += lane_xor<8>(ps);
+        if (c4 < n4 && (c4 & 11) == 0) ((float*)xsum)[2 * (c4 / 16) + ((c4 >> 2) & 1)] = ps;
+    }
+    __syncthreads();
+    float xv[64];
+    const float4* xq = (const float4*)(xs + q * kQ4XStride);
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const float4 f = xq[i];
+        xv[4 * i] = f.x, xv[4 * i + 1] = f.y, xv[4 * i + 2] = f.z, xv[4 * i + 3] = f.w;
+    }
+    const float2 xm = xsum[q];
+    for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+        const uint32_t nr = min(P, M - tile * P), next = min(tile + gridDim.x, tiles - 1), rr = t / G;
+        const float v = q4_quarter(hd, q0, q1, g, xv, xm), y0 = yp;
+        load(next);
+        load_y(next);
+        rd[ph0 < P ? ph * nq + q : P * nq] = v;  // padding threads: the spare slot
+        __syncthreads();
+        float a = 0.0f;
+        if (rr < nr)
+            for (uint32_t c = t % G; c < nq; c += G) a += rd[rr * nq + c];
+        a = sum_group(a, G);
+        if (t % G == 0 && rr < nr) y[tile * P + rr] = y0 + a;
+        float* const sw = rd;
+        rd = other, other = sw;
+    }
+}
+
+// The walking kernel for this shape, or EC_ERR_UNSUPPORTED.  G: lanes per row
+// sum of the kernel it stands in for.
+int launch_q4_f32_walk(hipStream_t st, const uint8_t* W, const float* x, float* y, uint32_t M, uint32_t nsb,
+                       uint32_t G) {
+    const uint32_t nq = 4 * nsb, room = nq <= 128 ? 256 : kWalkThreads, P = room / nq;
+    if (P == 0) return EC_ERR_UNSUPPORTED;
+    const uint32_t T = nq <= 128 ? 256 : (P * nq + 63) / 64 * 64;
+    // four 256-thread workgroups per CU, two larger ones; from three tiles each
+    // on (18432 x 2560: 9.8 us, 10.2 without; 9216 x 2560: 8.3 / 7.4)
+    const uint32_t tiles = (M + P - 1) / P, slots = nq <= 128 ? 1024 : 512;
+    if (tiles < 3 * slots || P * G > T) return EC_ERR_UNSUPPORTED;
+    uint32_t xpt = 1;
+    while (xpt * T < 16 * nq) xpt *= 2;
+    const uint32_t mg = (uint32_t)((((uint64_t)1 << 32) + nq - 1) / nq);
+    const size_t lds = ((size_t)nq * (kQ4XStride + 2) + 2 * ((size_t)P * nq + 1)) * 4;
+    if (lds > 160 * 1024) return EC_ERR_UNSUPPORTED;
+    switch (xpt * 100 + G) {
+#define EC_WALK(X, GG)                                                                                              \
+    case X * 100 + GG:                                                                                              \
+        hipLaunchKernelGGL((k_gguf_q4_K_f32_walk<X, GG>), dim3(slots), dim3(T), lds, st, W, x, y, M, nsb, P, mg); \
+        return EC_OK;
+        EC_WALK(1, 16) EC_WALK(1, 32) EC_WALK(1, 64) EC_WALK(2, 16) EC_WALK(2, 32) EC_WALK(2, 64)
+        EC_WALK(4, 16) EC_WALK(4, 32) EC_WALK(4, 64) EC_WALK(8, 16) EC_WALK(8, 32) EC_WALK(8, 64)
+#undef EC_WALK
+        default: return EC_ERR_UNSUPPORTED;
+    }
 }
 
 template <int RPT>
@@ -439,6 +545,11 @@ int gguf_mv_fast(int fmt, const uint8_t* W, const float* x, float* y, uint32_t M
         uint32_t xpt = 1;
         while (xpt * T < 16 * nq) xpt *= 2;
         if (T > 1024 || R > T || lds > 160 * 1024 || xpt > 16) return EC_ERR_UNSUPPORTED;
+        if (rpt == 1 && !p_env && !rpt_env) {
+            uint32_t G = 64;
+            while (G * P > T) G /= 2;
+            if (launch_q4_f32_walk(st, W, x, y, M, nsb, G) == EC_OK) return EC_OK;
+        }
         return launch_q4_f32(rpt, xpt, grid, blk, lds, st, W, x, y, M, nsb, P, R);
     }
     return EC_ERR_UNSUPPORTED;

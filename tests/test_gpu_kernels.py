@@ -592,3 +592,26 @@ def test_gguf_f32_matvec_full_shapes(hip, oc, fmt, N, K):
     hip.matvec_gguf_f32(fmt, dev(W), dev(x), y, N, K)
     ref = (oc.matvec_q8_0 if fmt == 6 else oc.matvec_q4_K)(W, x, y0)
     assert rel_l2(host(y), ref) < 1e-5
+
+
+@pytest.mark.parametrize("N,K", [(18437, 2560), (18432, 2560), (49170, 1024), (36865, 1536), (12289, 4096), (6147, 8192),
+                                 (6150, 9216), (6145, 10240)])
+def test_gguf_f32_q4_many_rows(hip, N, K):
+    """Q4_K matvecs from the size where workgroups walk over the rows (three tiles of P rows for each of 1024, at
+    K > 8192 512, workgroups): a row's sum is the bits of the same row in a call too short to walk, the first of which
+    are held to the oracle above; ragged last tiles, padding lanes (1536, 10240), y accumulated."""
+    import torch
+    from echohip.lib import Q4_K
+    g = torch.Generator(device="cuda").manual_seed(N)
+    W = torch.randint(0, 256, (N, K // 256, 144), generator=g, device="cuda", dtype=torch.int32).to(torch.uint8)
+    d = torch.rand((N, K // 256, 2), generator=g, device="cuda") * 0.01
+    W[:, :, :4] = d.half().view(torch.uint8)
+    x = torch.randn(K, generator=g, device="cuda")
+    y0 = torch.randn(N, generator=g, device="cuda")
+    y, ref = y0.clone(), y0.clone()
+    hip.matvec_gguf_f32(Q4_K, W, x, y, N, K)
+    part = N // 3 + 1  # too short to walk, long enough for one row per thread
+    for r in range(0, N, part):
+        n = min(part, N - r)
+        hip.matvec_gguf_f32(Q4_K, W[r:r + n].contiguous(), x, ref[r:r + n], n, K)
+    assert torch.equal(y.view(torch.int32), ref.view(torch.int32))
