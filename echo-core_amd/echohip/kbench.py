@@ -303,7 +303,7 @@ def gemm_case(hip, fmt, N, K, M=512, iters=20, seed=0):
     tops = ops / (mean_us * 1e-6) / 1e12
     del tiled
     torch.cuda.empty_cache()
-    return {"kernel": "k_gemm_q8_0" if fmt == L.Q8_0 else "k_gemm_q4_K", "M": M, "N": N, "K": K,
+    return {"kernel": "k_gemm Q8_0" if fmt == L.Q8_0 else "k_gemm Q4_K", "M": M, "N": N, "K": K,
             "us": round(mean_us, 2), "TOPs": round(tops, 1), "frac": round(tops / INT8_PEAK_TOPS, 4)}
 
 
